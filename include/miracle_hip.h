@@ -226,8 +226,9 @@ MR_API int mr_model_generate_greedy(mr_model *model, int max_new, int eos, int32
  * on each other's results, so they must all be resident at once: a plain
  * launch whose grid equals the CU count and whose registers fill a CU places
  * one on every CU when the GPU is otherwise idle.  If other work holds CUs and
- * a wait times out, the step fails with MR_ERR_TIMEOUT and the model switches to
- * MR_STEP_GRAPH at the next mr_model_reset (mr_model_get_step_mode reports it).
+ * a wait times out, the step fails with MR_ERR_TIMEOUT, and so does every later
+ * forward, greedy loop and traced step, whatever the mode, until mr_model_reset,
+ * which switches the model to MR_STEP_GRAPH (mr_model_get_step_mode reports it).
  * MR_STEP_GRAPH: six fused kernels per layer, replayed from a captured
  * hipGraph.  MR_STEP_EAGER: the same kernels launched one by one (for
  * profilers). */

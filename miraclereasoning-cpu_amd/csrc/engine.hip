@@ -787,6 +787,13 @@ int check_step_error(mr_model *m, const int *known = nullptr) {
     return MR_OK;
 }
 
+// After a timeout the device's position and rings have moved past the
+// model's, whatever step mode comes next: nothing runs until mr_model_reset.
+int check_sequence(mr_model *m, const char *what) {
+    if (!m->timed_out) return MR_OK;
+    return fail(MR_ERR_TIMEOUT, std::string(what) + ": a step of this sequence timed out; reset the model");
+}
+
 // Phase program of one step for the persistent kernel (GQA families).  Each
 // read names the phase whose cells it expects: x_phase for the input,
 // res_phase for a residual's previous value.
@@ -2259,6 +2266,7 @@ int prefill_batched(mr_model *m, int n, bool all, float *logits) {
 
 int mr_model_forward(mr_model *m, const int32_t *ids, int n, int flags, float *logits) {
     MR_TRY(check_ctx(m, "forward"));
+    MR_TRY(check_sequence(m, "forward"));
     MR_REQUIRE(ids && n > 0, "forward: input_ids must be a non-empty 1D integer sequence");
     const mr_model_desc &d = m->d;
     for (int i = 0; i < n; ++i)
@@ -2297,6 +2305,7 @@ int mr_model_forward(mr_model *m, const int32_t *ids, int n, int flags, float *l
 
 int mr_model_generate_greedy(mr_model *m, int max_new, int eos, int32_t *tokens, int *produced) {
     MR_TRY(check_ctx(m, "generate"));
+    MR_TRY(check_sequence(m, "generate"));
     MR_REQUIRE(tokens && produced && max_new >= 1, "generate: bad arguments");
     MR_REQUIRE(m->position >= 1, "generate: call forward first");
     MR_REQUIRE(m->position + max_new - 1 <= m->d.context_length, "generate: exceeds context_length");
@@ -2386,6 +2395,7 @@ int mr_model_choices(mr_model *m, int32_t *out, int64_t capacity, int *per_posit
 
 int mr_model_trace_step(mr_model *m, uint64_t *out, int64_t capacity, int *phases, int *grid) {
     MR_TRY(check_ctx(m, "trace_step"));
+    MR_TRY(check_sequence(m, "trace_step"));
     MR_REQUIRE(out && phases && grid, "trace_step: null argument");
     if (!m->persistent_ok || m->mode != MR_STEP_PERSISTENT)
         return fail(MR_ERR_STATE, "trace_step: the model does not run the persistent step kernel");

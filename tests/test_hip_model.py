@@ -428,6 +428,38 @@ def test_step_timeout_falls_back_to_graph_mode(backend):
     model.close()
 
 
+@pytest.mark.parametrize("then", ["persistent", "graph", "eager", "graph, then persistent"])
+def test_timed_out_sequence_fails_until_reset(backend, then):
+    """Through the engine (the C ABI, below MiracleModel's own failed flag):
+    after a timed-out step, whose tokens have moved the device's position and
+    not the model's, a forward by tokens or by batch, a greedy loop and a traced
+    step report the timeout in every step mode, until mr_model_reset."""
+    from miracle_hip import HIPError
+    from miracle_hip.model import FWD_BATCHED
+    wl = presets.workload("flashnano-1.5-tiny")
+    weights = synthetic.synthetic_weights(wl["config"], wl["seed"], wl["dtype"])
+    model = MiracleModel(ModelConfig.from_dict(wl["config"]), weights, backend=backend, context_length=64)
+    engine, ids = model.engine, [5, 9, 2, 7, 11, 3]
+    engine.set_step_mode("persistent")
+    want = engine.forward(ids, 0)
+    engine.reset()
+    engine.forward(ids[:2], 0)
+    engine.debug_step_timeout()
+    with pytest.raises(HIPError, match="timed out"):
+        engine.forward(ids[2:4], 0)
+    assert engine.position() == 2
+    for mode in then.split(", then "):
+        engine.set_step_mode(mode)
+    for call in (lambda: engine.forward(ids[2:4], FWD_BATCHED), lambda: engine.forward(ids[2:3], 0),
+                 lambda: engine.generate_greedy(4, 0), lambda: engine.trace_step()):
+        with pytest.raises(HIPError, match="timed out"):
+            call()
+    assert engine.position() == 2
+    engine.reset()
+    np.testing.assert_allclose(engine.forward(ids, 0), want, atol=2e-5, rtol=2e-4)
+    model.close()
+
+
 def test_weight_cache_budget_and_untied_head(backend):
     # reference tests/test_inference.py:72-84: a 4 KiB weight budget gives the
     # same logits (here every weight is resident in HBM whatever the budget)

@@ -985,21 +985,8 @@ int setup_persistent(mr_model *m) {
 // per-inner-loop rings (capacity = context) and block sums, expert table.
 // FP16 copies of projection matrices for the batched prefill's FP16-term
 // GEMMs (gemm.h), each with its power-of-two scale; the matrices in `shared`
-// (a SwiGLU pair, one tile holds rows of both) take their smaller scale.  F16
-// matrices, which the term products also take as they are (in about twice the
-// time), get copies only while a quarter of the device's memory stays free: a
-// model that fills the device runs without them.
+// (a SwiGLU pair, one tile holds rows of both) take their smaller scale.
 int f16_copies(mr_model *m, std::initializer_list<Weight *> ws, std::initializer_list<Weight *> shared) {
-    size_t need = 0, free_bytes = 0, total_bytes = 0;
-    for (Weight *w : ws)
-        if (w->dtype == MR_F16) need += (size_t)w->rows * w->cols * 2;
-    if (need) {
-        MR_HIP(hipMemGetInfo(&free_bytes, &total_bytes), "device memory");
-        if (free_bytes < need + total_bytes / 4) {
-            for (Weight *w : ws) w->f16_scale = 0.0f;
-            return MR_OK;
-        }
-    }
     for (Weight *w : ws)
         MR_TRY(gemm_f16_weight_scale(m->ctx->stream, w->ptr, w->dtype, w->rows * w->cols, &w->f16_scale));
     float common = INFINITY;
@@ -1008,7 +995,7 @@ int f16_copies(mr_model *m, std::initializer_list<Weight *> ws, std::initializer
     for (Weight *w : ws)
         if (w->f16_scale > 0.0f) {
             MR_TRY(device_alloc(m, (size_t)w->rows * w->cols * 2, &w->f16));
-            MR_TRY(gemm_f16_weight_copy(m->ctx->stream, w->ptr, w->dtype, w->rows * w->cols, w->f16_scale, w->f16));
+            MR_TRY(gemm_f16_weight_copy(m->ctx->stream, w->ptr, w->rows * w->cols, w->f16_scale, w->f16));
         }
     return MR_OK;
 }
@@ -1612,6 +1599,7 @@ struct PrefillWs {
     float *act_scale = nullptr;  // row scales of the SwiGLU output written in FP16 terms (into act)
     float *att_scale = nullptr;  // row scales of the attended values written in FP16 terms (into att)
     _Float16 *planes = nullptr;  // and its hi and lo FP16 planes
+    bool planes3 = false;        // F16 weights: with room for three BF16 planes (GemmArgs::planes3)
     float *part = nullptr;       // and the sums of their K slices (GemmArgs::part)
     _Float16 *kv16 = nullptr;    // attention: the attended keys and values in FP16 terms
     int kv16_rows = 0;
@@ -1637,6 +1625,12 @@ int prefill_workspace(mr_model *m, int rows, bool all, PrefillWs *w) {
     // rows split into FP16 terms at once: a chunk, its pooled CBR rows, or its
     // rows gathered for every expert slot
     const size_t split_rows = std::max({r, pr, heavy ? r * slots : 0});
+    w->planes3 = false;
+    if (!heavy)
+        for (const Layer &L : m->layers)
+            for (const Weight *t : {&L.qkv, &L.kv_up, &L.o, &L.ffn.gate, &L.ffn.down})
+                w->planes3 |= t->ptr && t->dtype == MR_F16;
+    const size_t split_width = std::max({h, qd, (size_t)d.ffn_dim});
     int max_cap = 0;
     for (const Layer &L : m->layers) max_cap = std::max(max_cap, L.capacity);
     for (const Layer &L : m->layers) max_cap = std::max(max_cap, L.light_cap);
@@ -1671,7 +1665,7 @@ int prefill_workspace(mr_model *m, int rows, bool all, PrefillWs *w) {
         // flashnano-1.6
         {(void **)&w->cbr_scores, pr * (cbr ? d.cbr_chunk_size : 0)}, {(void **)&w->cbr_pooled, pr * h}, {(void **)&w->cbr_anchor, pr}, {(void **)&w->cbr_kv, pr * 2 * kvw},
         {(void **)&w->rowscale, split_rows}, {(void **)&w->act_scale, r}, {(void **)&w->att_scale, r},
-        {(void **)&w->planes, split_rows * std::max({h, qd, (size_t)d.ffn_dim})}, {(void **)&w->part, kGemmPartFloats},
+        {(void **)&w->planes, split_rows * split_width * (w->planes3 ? 3 : 2) / 2}, {(void **)&w->part, kGemmPartFloats},
         {(void **)&w->kv16, kv16}, {(void **)&w->kv16_scale, 2 * kvw}, {(void **)&w->kv16_max, 2 * kvw},
         {(void **)&w->kv_part, (size_t)w->kv_part_blocks * 2 * max_kvh}};
     auto up = [](size_t floats) { return (floats + 63) & ~(size_t)63; };   // 256-byte slices
@@ -1804,7 +1798,7 @@ int cbr_layer_rows(mr_model *m, Layer &L, const PrefillWs &w, int p0, int T) {
         kv.a = w.cbr_pooled; kv.lda = h; kv.dtype = L.qkv.dtype;
         kv.w = (const char *)L.qkv.ptr + (size_t)qd * h * dtype_bytes(L.qkv.dtype);
         kv.c = w.cbr_kv; kv.ldc = 2 * kvw; kv.m = nc * slots; kv.n = 2 * kvw; kv.k = h;
-        kv.wscale = L.qkv.f16_scale; kv.ascale = w.rowscale; kv.ahl_ws = w.planes; kv.part = w.part;
+        kv.wscale = L.qkv.f16_scale; kv.ascale = w.rowscale; kv.ahl_ws = w.planes; kv.part = w.part; kv.planes3 = w.planes3;
         if (L.qkv.f16) kv.wh = (const _Float16 *)L.qkv.f16 + (size_t)qd * h;
         MR_TRY(launch_gemm(s, GEMM_STORE, kv));
         k_cbr_finish_rows<<<nc * slots, 256, (size_t)kvw * sizeof(float), s>>>(
@@ -1830,6 +1824,7 @@ int gqa_layer_rows(mr_model *m, Layer &L, const Layer *next, const PrefillWs &w,
     g.a = w.xn; g.lda = h; g.w = L.qkv.ptr; g.dtype = L.qkv.dtype; g.c = w.qkv; g.ldc = ld;
     g.m = T; g.n = ld; g.k = h; g.wscale = L.qkv.f16_scale; g.wh = L.qkv.f16; g.ascale = w.rowscale; g.ahl_ws = w.planes;
     g.part = w.part;
+    g.planes3 = w.planes3;
     // the normalized rows go straight into the FP16-term GEMM's A workspace
     // (flashnano-1.6 pools them in FP32 first)
     const bool cbr = d.family == MR_FAMILY_FLASHNANO_16;
@@ -1864,7 +1859,7 @@ int gqa_layer_rows(mr_model *m, Layer &L, const Layer *next, const PrefillWs &w,
     }
     // the attended values straight into the O projection's FP16 terms (att
     // holds T x qd floats, the same bytes as its two planes of halves)
-    const bool att_split = !a.ext && L.o.f16_scale > 0.0f && prefill_attention_presplit(a);
+    const bool att_split = !a.ext && L.o.dtype == MR_BF16 && L.o.f16_scale > 0.0f && prefill_attention_presplit(a);
     if (att_split) {
         a.out_hl = (_Float16 *)w.att;
         a.out_scale = w.att_scale;
@@ -1879,6 +1874,7 @@ int gqa_layer_rows(mr_model *m, Layer &L, const Layer *next, const PrefillWs &w,
     o.a = w.att; o.lda = qd; o.w = L.o.ptr; o.dtype = L.o.dtype; o.c = w.x; o.ldc = h;
     o.m = T; o.n = h; o.k = qd; o.scale = d.residual_scale; o.wscale = L.o.f16_scale; o.wh = L.o.f16;
     o.part = w.part;
+    o.planes3 = w.planes3;
     o.ascale = att_split ? w.att_scale : w.rowscale;
     o.ahl_ws = att_split ? (_Float16 *)w.att : w.planes;
     o.a_split = att_split;
@@ -1888,6 +1884,7 @@ int gqa_layer_rows(mr_model *m, Layer &L, const Layer *next, const PrefillWs &w,
     gu.wscale = L.ffn.gate.f16_scale; gu.wh = L.ffn.gate.f16; gu.wh2 = L.ffn.up.f16; gu.ascale = w.rowscale;
     gu.ahl_ws = w.planes;
     gu.part = w.part;
+    gu.planes3 = w.planes3;
     gu.a_split = gu.wscale > 0.0f && rms_split_fits(h);
     // the SwiGLU output straight into the down projection's FP16 terms (act
     // holds T x ffn floats, the same bytes as its two planes of halves)
@@ -1912,6 +1909,7 @@ int gqa_layer_rows(mr_model *m, Layer &L, const Layer *next, const PrefillWs &w,
     dn.m = T; dn.n = h; dn.k = ffn; dn.scale = d.residual_scale; dn.wscale = L.ffn.down.f16_scale;
     dn.wh = L.ffn.down.f16;
     dn.part = w.part;
+    dn.planes3 = w.planes3;
     dn.ascale = act_split ? w.act_scale : w.rowscale;
     dn.ahl_ws = act_split ? (_Float16 *)w.act : w.planes;
     dn.a_split = act_split;
@@ -2060,8 +2058,8 @@ int light_layer_rows(mr_model *m, Layer &L, const PrefillWs &w, const LightPlan 
     // the normalized rows straight into FP16 terms where the Q/latent and FFN
     // GEMMs take them (BF16 weights with FP16 copies), with the scales of the
     // SwiGLU output for the down projection's FP16 terms
-    const bool xn_split = L.qkv.f16_scale > 0.0f && rms_split_fits(h);
-    const bool gu_split = xn_split && L.ffn.gate.f16_scale > 0.0f;
+    const bool xn_split = L.qkv.dtype == MR_BF16 && L.qkv.f16_scale > 0.0f && rms_split_fits(h);
+    const bool gu_split = xn_split && L.ffn.gate.dtype == MR_BF16 && L.ffn.gate.f16_scale > 0.0f;
     const bool act_split = gu_split && act_split_fits(L.ffn, h);
     if (!gu_split) MR_TRY(launch_rms_rows(s, w.x, h, L.a_norm.f(), d.norm_eps, h, w.xn, h, T));
     if (xn_split)
@@ -2073,6 +2071,7 @@ int light_layer_rows(mr_model *m, Layer &L, const PrefillWs &w, const LightPlan 
         g.wh = wt.f16 ? (const void *)((const _Float16 *)wt.f16 + row0 * wt.cols) : nullptr;
         g.ascale = w.rowscale;
         g.part = w.part;
+        g.planes3 = w.planes3;
         g.ahl_ws = w.planes;
     };
     GemmArgs q;   // the Q rows of the packed [Wq; Wlatent]
@@ -2133,7 +2132,7 @@ int light_layer_rows(mr_model *m, Layer &L, const PrefillWs &w, const LightPlan 
     a.kv16 = w.kv16; a.kv16_rows = w.kv16_rows; a.kv16_scale = w.kv16_scale; a.kv16_max = w.kv16_max;
     a.kv_part = w.kv_part; a.kv_part_blocks = w.kv_part_blocks;
     // without an extra partial, the attended values straight into the O projection's FP16 terms
-    const bool att_split = !a.ext && L.o.f16_scale > 0.0f && prefill_attention_presplit(a);
+    const bool att_split = !a.ext && L.o.dtype == MR_BF16 && L.o.f16_scale > 0.0f && prefill_attention_presplit(a);
     if (att_split) {
         a.out_hl = (_Float16 *)w.att;
         a.out_scale = w.att_scale;

@@ -8,7 +8,7 @@
 // weights are BF16 (one term), F16 (two terms, exact: 11 significant bits fit
 // in hi + lo) or FP32 (three terms).  Products of terms whose orders sum to
 // at most 2 are accumulated (3, 5 or 6 MFMAs per tile step), so the result
-// carries FP32-level error.  FP16 scheme (16-bit weights): each activation row
+// carries FP32-level error.  FP16 scheme (BF16 weights): each activation row
 // is scaled by a power of two into FP16 range and carried as hi + lo FP16
 // terms (about 2^-23 of its value left behind), the weights scaled by a power
 // of two are exact in FP16, and two MFMAs per tile step carry the product.
@@ -30,7 +30,7 @@ struct GemmArgs {
     int ldc = 0;
     int m = 0, n = 0, k = 0;     // GEMM_SWIGLU: n = output columns (FFN width)
     float scale = 1.0f;          // GEMM_RESIDUAL: c += scale * (A . W^T)
-    // FP16 terms (16-bit weights only): wscale > 0 is the weights' power-of-two
+    // FP16 terms (BF16 weights only): wscale > 0 is the weights' power-of-two
     // scale into FP16 range (gemm_f16_weight_scale) and wh (wh2: SwiGLU up
     // rows) the weights converted with it; ascale (m floats) and ahl_ws
     // (2 m k halves) are device workspaces that receive A's row scales and its
@@ -58,6 +58,10 @@ struct GemmArgs {
     // here, for the caller's next kernel to add up in order with what it does
     // to the row anyway; 0 where c is written as always.
     int *left = nullptr;
+    // F16 weights: ahl_ws has room for three planes (3 m k halves; ascale as
+    // above), so the rows may be split once, into BF16 terms, for products whose
+    // operands are copied into LDS (without, k_gemm splits them in every tile).
+    bool planes3 = false;
 };
 constexpr size_t kGemmPartFloats = (size_t)5 << 20;   // two 64 x 128 tiles for each of 256 CUs, and room
 
@@ -81,21 +85,20 @@ int launch_row_split(hipStream_t s, const float *a, int lda, int m, int k, float
 // output columns over many rows, where the plain GEMM has too few tiles.
 int launch_gemm_split(hipStream_t s, const GemmArgs &g, int slices, float *part);
 
-// The power of two 2^s that puts max |w| of a BF16 or F16 matrix of `count`
-// values in [2^13, 2^14) (1 for an all-zero matrix), so that w 2^s is exact in
-// FP16 for every |w| >= 2^-31 max |w| (F16: 2^-28); 0 for a matrix holding a non-finite value or
+// The power of two 2^s that puts max |w| of a BF16 matrix of `count` values
+// in [2^13, 2^14) (1 for an all-zero matrix), so that w 2^s is exact in FP16
+// for every |w| >= 2^-31 max |w|; 0 for a matrix holding a non-finite value or
 // another dtype (the FP16 scheme is then not used).  Synchronizes the stream.
 int gemm_f16_weight_scale(hipStream_t s, const void *w, int dtype, int64_t count, float *scale);
 
 // An upper bound on the largest row norm, max_r sqrt(sum_k w[r][k]^2), of a
-// 16-bit matrix of `rows` x `cols` values into *norm (0 for another dtype or a
+// BF16 matrix of `rows` x `cols` values into *norm (0 for another dtype or a
 // non-finite value).  Synchronizes the stream.
 int gemm_row_norm_bound(hipStream_t s, const void *w, int dtype, int64_t rows, int64_t cols, float *norm);
 
-// dst[i] = FP16(w[i] * scale) for `count` BF16 or F16 values (exact for a scale
-// from gemm_f16_weight_scale, or a smaller power of two, down to the values
-// named there).
-int gemm_f16_weight_copy(hipStream_t s, const void *w, int dtype, int64_t count, float scale, void *dst);
+// dst[i] = FP16(w[i] * scale) for `count` BF16 values (exact for a scale from
+// gemm_f16_weight_scale, or a smaller power of two).
+int gemm_f16_weight_copy(hipStream_t s, const void *w, int64_t count, float scale, void *dst);
 
 // Groups of rows with their own weights (the experts of a batched MoE), one
 // launch: group z multiplies rows offset[z] .. offset[z] + count[z] of g.a by

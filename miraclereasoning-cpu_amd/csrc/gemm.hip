@@ -148,6 +148,16 @@ __device__ __forceinline__ void split2h(float x, _Float16 &hi, _Float16 &lo) {
     lo = (_Float16)(x - (float)hi);
 }
 
+// Eight halves as two BF16 terms each (exact: 11 bits fit in 8 + 8).
+__device__ __forceinline__ void split_f16(const f16x8 &f, bf16x8 &hi, bf16x8 &lo) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float x = (float)f[e];
+        hi[e] = (__bf16)x;
+        lo[e] = (__bf16)(x - (float)hi[e]);
+    }
+}
+
 template <int DT>
 __device__ __forceinline__ void store_w(__bf16 (*bs)[kBN][kPitch], const WRegs<DT> &r) {
     const int tid = threadIdx.x;
@@ -161,14 +171,8 @@ __device__ __forceinline__ void store_w(__bf16 (*bs)[kBN][kPitch], const WRegs<D
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int idx = tid + kThreads * i;
-            const f16x8 f = __builtin_bit_cast(f16x8, r.v[i]);
             bf16x8 h, l;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float x = (float)f[e];
-                h[e] = (__bf16)x;
-                l[e] = (__bf16)(x - (float)h[e]);
-            }
+            split_f16(__builtin_bit_cast(f16x8, r.v[i]), h, l);
             *(bf16x8 *)&bs[0][idx >> 2][(idx & 3) * 8] = h;
             *(bf16x8 *)&bs[1][idx >> 2][(idx & 3) * 8] = l;
         }
@@ -204,31 +208,30 @@ __device__ __forceinline__ f32x4 mfma(const f16x8 &a, const f16x8 &b, const f32x
 
 // What the LDS-copy tile multiplies.  kModelTerms: A in two FP16 planes by the
 // model's FP16 weight copies (their scale in g.wscale).  kF16Rows, kBF16Rows:
-// single products by weights as they are stored, F16 (A in two FP16 planes) or
-// BF16 (three BF16 planes: 24 bits).  Splitting a value into terms turns an
-// infinity into inf - inf, and a scaled row can overflow where its FP32
-// products would not, so single products that come out non-finite are summed
-// again in plain FP32.
-//
-// The matrix cores align a product of a subnormal half by the exponent of the
-// smallest normal one and lose its last bits (a row of weights near 2^-22 came
-// out 2^-19 off), so F16 weights are multiplied by 2^8 in registers (exact;
-// those above 255 overflow and are summed again).
+// weights as they are stored by A in three BF16 planes, which keep 24 bits of
+// every value however small it is beside its row's largest (two FP16 planes
+// keep them relative to the row's largest only); a BF16 weight is one term, an
+// F16 weight two BF16 terms split in registers (exact, subnormals too, which
+// the FP16 matrix cores would multiply at fewer bits).  4096 rows of 5632 x
+// 2048 take 283 us by BF16 weights (three products a weight) and 437 by F16
+// weights (five); in two FP16 planes 213.
+// Splitting a value into terms turns an infinity into inf - inf, and a scaled
+// row can overflow where its FP32 products would not, so STORE products of
+// these that come out non-finite are summed again in plain FP32.
 enum { kModelTerms = 0, kF16Rows = 1, kBF16Rows = 2 };
-constexpr float kF16RowsScale = 256.0f;
 template <int SCH>
 struct Terms {
-    typedef _Float16 H;
-    typedef f16x8 V;
-    static constexpr int kPlanes = 2;
-    static constexpr bool kRecompute = SCH == kF16Rows;
-};
-template <>
-struct Terms<kBF16Rows> {
     typedef __bf16 H;
     typedef bf16x8 V;
-    static constexpr int kPlanes = 3;
+    static constexpr int kPlanes = 3, kWeightTerms = SCH == kF16Rows ? 2 : 1;
     static constexpr bool kRecompute = true;
+};
+template <>
+struct Terms<kModelTerms> {
+    typedef _Float16 H;
+    typedef f16x8 V;
+    static constexpr int kPlanes = 2, kWeightTerms = 1;
+    static constexpr bool kRecompute = false;
 };
 
 // Output (row, col) of g from its FP32 rows and stored weights, k in order.
@@ -331,8 +334,7 @@ __device__ __forceinline__ void gemm_store(const GemmArgs &g, int m0, int n0, co
             }
         }
     }
-    if constexpr (Terms<SCH>::kRecompute) {
-        static_assert(EPI == GEMM_STORE, "plain products only");
+    if constexpr (Terms<SCH>::kRecompute && EPI == GEMM_STORE) {
         if (bad)
 #pragma unroll 1
             for (int i = 0; i < 4 * MI * NI; ++i) {
@@ -588,7 +590,7 @@ __device__ __forceinline__ void gemm_tile_hd(const GemmArgs &g, int m0, int n0, 
                                              float *part = nullptr) {
     typedef typename Terms<SCH>::H H;
     typedef typename Terms<SCH>::V V;
-    constexpr int P = Terms<SCH>::kPlanes;
+    constexpr int P = Terms<SCH>::kPlanes, T = Terms<SCH>::kWeightTerms;
     static_assert(KB == 32 || KB == 64, "k-step");
     constexpr int BM = 32 * MI;                    // rows of A
     constexpr int CPR = KB / 8;                    // 16-byte chunks per row
@@ -670,12 +672,13 @@ __device__ __forceinline__ void gemm_tile_hd(const GemmArgs &g, int m0, int n0, 
 #pragma unroll
         for (int kk = 0; kk < KB / 32; ++kk) {
             const int c = 4 * kk + lq;
-            V bf[NI];
+            V bf[T][NI];
 #pragma unroll
             for (int ni = 0; ni < NI; ++ni) {
                 const int r = wn * 16 * NI + ni * 16 + lr;
-                bf[ni] = *(const V *)(ws + r * KB + (c ^ chunk_swizzle<KB>(r)) * 8);
-                if constexpr (SCH == kF16Rows) bf[ni] *= (_Float16)kF16RowsScale;
+                const H *wp = ws + r * KB + (c ^ chunk_swizzle<KB>(r)) * 8;
+                if constexpr (SCH == kF16Rows) split_f16(*(const f16x8 *)wp, bf[0][ni], bf[1][ni]);
+                else bf[0][ni] = *(const V *)wp;
             }
 #pragma unroll
             for (int mi = 0; mi < MI; ++mi) {
@@ -683,11 +686,15 @@ __device__ __forceinline__ void gemm_tile_hd(const GemmArgs &g, int m0, int n0, 
                 V term[P];
 #pragma unroll
                 for (int p = P - 1; p >= 0; --p) term[p] = *(const V *)(ah + p * SA + off);
-                // the smallest term first
+                // term pairs (A order, W order) with orders summing to <= 2, smallest first
 #pragma unroll
-                for (int p = P - 1; p >= 0; --p)
+                for (int o = 2; o >= 0; --o)
 #pragma unroll
-                    for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = mfma(term[p], bf[ni], acc[mi][ni]);
+                    for (int q = T - 1; q >= 0; --q)
+                        if (o - q >= 0 && o - q < P)
+#pragma unroll
+                            for (int ni = 0; ni < NI; ++ni)
+                                acc[mi][ni] = mfma(term[o - q], bf[q][ni], acc[mi][ni]);
             }
         }
         if (S == 1 && kt + 1 < kt1) {
@@ -926,7 +933,7 @@ __global__ void __launch_bounds__(256) k_row_split_reg(const float *a, int lda, 
     }
 }
 
-// The three BF16 planes of kBF16Rows, one wave per row: row r's scale as
+// The three BF16 planes of kF16Rows and kBF16Rows, one wave per row: row r's scale as
 // above into scale[r], a[r][k] 2^t = hi + mid + lo into planes [3][m][k].
 __global__ void __launch_bounds__(256) k_row_split3(const float *a, int lda, int m, int k, float *scale, __bf16 *out) {
     const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -1181,34 +1188,32 @@ void row_split(hipStream_t s, const float *a, int lda, int m, int k, float *scal
     else k_row_split<<<ceil_div(m, 4), 256, 0, s>>>(a, lda, m, k, scale, hl);
 }
 
-template <int DT>
-__global__ void __launch_bounds__(256) k_to_f16(const uint16_t *w, int64_t count, float scale, _Float16 *dst) {
+__global__ void __launch_bounds__(256) k_bf16_to_f16(const uint16_t *w, int64_t count, float scale, _Float16 *dst) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x)
-        dst[i] = (_Float16)(mr::load_w<DT>(w, i) * scale);
+        dst[i] = (_Float16)(__uint_as_float((unsigned)w[i] << 16) * scale);
 }
 
-// max |w| over an array of 16-bit values as the bits of a non-negative float
-// (atomic max on the bit patterns, which order like the values).
-template <int DT>
-__global__ void __launch_bounds__(256) k_abs_max(const uint16_t *w, int64_t count, unsigned *out) {
+// max |w| over a BF16 array as the bits of a non-negative float (atomic max
+// on the bit patterns, which order like the values).
+__global__ void __launch_bounds__(256) k_abs_max_bf16(const uint16_t *w, int64_t count, unsigned *out) {
     unsigned mx = 0;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x)
-        mx = max(mx, __float_as_uint(mr::load_w<DT>(w, i)) & 0x7fffffffu);
+        mx = max(mx, (unsigned)(w[i] & 0x7fffu) << 16);
     for (int off = 32; off > 0; off >>= 1) mx = max(mx, (unsigned)__shfl_xor((int)mx, off));
     if ((threadIdx.x & 63) == 0) atomicMax(out, mx);
 }
 
 // max over rows of the row's L2 norm, one wave per row, as the bits of a
 // non-negative float (atomic max on the bit patterns).
-template <int DT>
-__global__ void __launch_bounds__(256) k_row_norm_max(const uint16_t *w, int64_t rows, int64_t cols, unsigned *out) {
+__global__ void __launch_bounds__(256) k_row_norm_max_bf16(const uint16_t *w, int64_t rows, int64_t cols,
+                                                           unsigned *out) {
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
     const uint16_t *r = w + row * cols;
     float ss = 0.0f;
     for (int64_t c = lane; c < cols; c += kWave) {
-        const float v = mr::load_w<DT>(r, c);
+        const float v = __uint_as_float((unsigned)r[c] << 16);
         ss += v * v;
     }
     ss = wave_sum(ss);
@@ -1340,7 +1345,7 @@ template <int DT>
 int launch_grouped_dt(hipStream_t s, int epi, const GemmArgs &g, const GemmGroups &gg) {
     const int cols = epi == GEMM_SWIGLU ? kBN / 2 : kBN;
     const dim3 grid(ceil_div(g.n, cols), ceil_div(gg.max_rows, kBM), gg.groups);
-    if (DT != MR_F32 && gg.wh) {
+    if (DT == MR_BF16 && gg.wh) {
         MR_REQUIRE(g.m > 0 && g.ascale && g.ahl_ws && gg.wscale && (epi != GEMM_SWIGLU || gg.wh2),
                    "grouped gemm: FP16 terms need the rows to split, their workspaces and the weights' scales");
         GemmArgs h = g;
@@ -1446,7 +1451,7 @@ template <int DT>
 int launch_dt(hipStream_t s, int epi, const GemmArgs &g) {
     const int cols = epi == GEMM_SWIGLU ? kBN / 2 : kBN;
     const dim3 grid(ceil_div(g.n, cols), ceil_div(g.m, kBM));
-    if (DT != MR_F32 && g.wscale > 0.0f) {
+    if (DT == MR_BF16 && g.wscale > 0.0f) {
         GemmArgs h = g;
         h.ahl = g.ahl_ws;
         h.w = g.wh;   // 16-bit rows: the BF16 loaders read them as they are
@@ -1471,6 +1476,26 @@ int launch_dt(hipStream_t s, int epi, const GemmArgs &g) {
         }
         MR_LAUNCHED("enqueue MFMA GEMM (FP16 terms)");
         return MR_OK;
+    }
+    // F16 weights as stored by three BF16 planes of the rows: the products of
+    // k_gemm<MR_F16> in its order, with K in slices and operands copied into LDS
+    // (prefill of four layers of flashnano-1.7, us by k_gemm -> here: 45 tokens
+    // 2582 -> 667, 217 2641 -> 1102, 1000 3164 -> 2429, 4096 7368 -> 6997).
+    if constexpr (DT == MR_F16) {
+        if (g.planes3 && !g.ldw && dma_tile_fits(g)) {
+            GemmArgs h = g;
+            h.ahl = g.ahl_ws;
+            h.wscale = 1.0f;
+            k_row_split3<<<ceil_div(g.m, 4), 256, 0, s>>>(g.a, g.lda, g.m, g.k, g.ascale, (__bf16 *)g.ahl_ws);
+            switch (epi) {
+                case GEMM_STORE: launch_hd<GEMM_STORE, kF16Rows>(s, h); break;
+                case GEMM_RESIDUAL: launch_hd<GEMM_RESIDUAL, kF16Rows>(s, h); break;
+                case GEMM_SWIGLU: launch_hd<GEMM_SWIGLU, kF16Rows>(s, h); break;
+                default: return fail(MR_ERR_INVALID, "gemm: unknown epilogue");
+            }
+            MR_LAUNCHED("enqueue MFMA GEMM (F16 weights, BF16 terms)");
+            return MR_OK;
+        }
     }
     // FP32 weights in few tiles: FP32 products on the FP32 matrix cores, K in
     // slices.  us in terms -> here at 2 x 2816 x 1024, 1024 x 2816: 32 rows 69.1
@@ -1548,16 +1573,14 @@ int launch_gemm_grouped(hipStream_t s, int epilogue, const GemmArgs &g, const Ge
 int gemm_f16_weight_scale(hipStream_t s, const void *w, int dtype, int64_t count, float *scale) {
     MR_REQUIRE(scale && (w || count == 0) && count >= 0, "f16 weight scale: bad arguments");
     *scale = 0.0f;
-    if (dtype == MR_F32 || count == 0) return MR_OK;
+    if (dtype != MR_BF16 || count == 0) return MR_OK;
     unsigned *dev = nullptr;
     MR_HIP(hipMalloc((void **)&dev, sizeof(unsigned)), "f16 weight scale");
     unsigned bits = 0;
     hipError_t e = hipMemsetAsync(dev, 0, sizeof(unsigned), s);
     if (e == hipSuccess) {
         const int64_t blocks = std::min<int64_t>(ceil_div(count, (int64_t)256 * 16), 4096);
-        const int grid = (int)std::max<int64_t>(blocks, 1);
-        if (dtype == MR_BF16) k_abs_max<MR_BF16><<<grid, 256, 0, s>>>((const uint16_t *)w, count, dev);
-        else k_abs_max<MR_F16><<<grid, 256, 0, s>>>((const uint16_t *)w, count, dev);
+        k_abs_max_bf16<<<(int)std::max<int64_t>(blocks, 1), 256, 0, s>>>((const uint16_t *)w, count, dev);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpyAsync(&bits, dev, sizeof(unsigned), hipMemcpyDeviceToHost, s);
@@ -1579,16 +1602,14 @@ int gemm_f16_weight_scale(hipStream_t s, const void *w, int dtype, int64_t count
 int gemm_row_norm_bound(hipStream_t s, const void *w, int dtype, int64_t rows, int64_t cols, float *norm) {
     MR_REQUIRE(norm && (w || rows * cols == 0) && rows >= 0 && cols >= 0, "row norm bound: bad arguments");
     *norm = 0.0f;
-    if (dtype == MR_F32 || rows == 0 || cols == 0) return MR_OK;
+    if (dtype != MR_BF16 || rows == 0 || cols == 0) return MR_OK;
     MR_REQUIRE(ceil_div(rows, (int64_t)4) <= INT32_MAX, "row norm bound: too many rows");
     unsigned *dev = nullptr;
     MR_HIP(hipMalloc((void **)&dev, sizeof(unsigned)), "row norm bound");
     unsigned bits = 0;
     hipError_t e = hipMemsetAsync(dev, 0, sizeof(unsigned), s);
     if (e == hipSuccess) {
-        const int grid = (int)ceil_div(rows, (int64_t)4);
-        if (dtype == MR_BF16) k_row_norm_max<MR_BF16><<<grid, 256, 0, s>>>((const uint16_t *)w, rows, cols, dev);
-        else k_row_norm_max<MR_F16><<<grid, 256, 0, s>>>((const uint16_t *)w, rows, cols, dev);
+        k_row_norm_max_bf16<<<(int)ceil_div(rows, (int64_t)4), 256, 0, s>>>((const uint16_t *)w, rows, cols, dev);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpyAsync(&bits, dev, sizeof(unsigned), hipMemcpyDeviceToHost, s);
@@ -1603,11 +1624,10 @@ int gemm_row_norm_bound(hipStream_t s, const void *w, int dtype, int64_t rows, i
     return MR_OK;
 }
 
-int gemm_f16_weight_copy(hipStream_t s, const void *w, int dtype, int64_t count, float scale, void *dst) {
-    MR_REQUIRE(w && dst && count > 0 && scale > 0.0f && dtype != MR_F32, "f16 weight copy: bad arguments");
+int gemm_f16_weight_copy(hipStream_t s, const void *w, int64_t count, float scale, void *dst) {
+    MR_REQUIRE(w && dst && count > 0 && scale > 0.0f, "f16 weight copy: bad arguments");
     const int64_t blocks = std::min<int64_t>(ceil_div(count, (int64_t)256 * 8), 8192);
-    if (dtype == MR_BF16) k_to_f16<MR_BF16><<<(int)blocks, 256, 0, s>>>((const uint16_t *)w, count, scale, (_Float16 *)dst);
-    else k_to_f16<MR_F16><<<(int)blocks, 256, 0, s>>>((const uint16_t *)w, count, scale, (_Float16 *)dst);
+    k_bf16_to_f16<<<(int)blocks, 256, 0, s>>>((const uint16_t *)w, count, scale, (_Float16 *)dst);
     MR_LAUNCHED("enqueue f16 weight copy");
     return MR_OK;
 }
@@ -1616,11 +1636,10 @@ int gemm_f16_weight_copy(hipStream_t s, const void *w, int dtype, int64_t count,
 //   - up to 8 rows, rows of whole 16-byte vectors: k_rows_gemv (up to 4 where
 //     the next path is open: 8 rows of 5632 x 2048 BF16 take 15.8 us there,
 //     12 take 13.2 in terms);
-//   - 16-bit weights, K a multiple of 64, 16-byte aligned: x in FP16 or BF16
-//     terms once (k_row_split, k_row_split3), then the LDS-copy tiles over the
-//     weights as stored.  Against 64 x 64 FP32 tiles: 333 rows of 5632 x 2048
-//     BF16 346 -> 46 us, of 2048 x 5632 894 -> 47; 50 rows of 2816 x 1024 F16
-//     142 -> 11.4;
+//   - 16-bit weights, K a multiple of 64, 16-byte aligned: x in three BF16
+//     terms once (k_row_split3), then the LDS-copy tiles over the weights as
+//     stored.  Against 64 x 64 FP32 tiles: 333 rows of 5632 x 2048 BF16 346 ->
+//     46 us, of 2048 x 5632 894 -> 47; F16 348 -> 85 and 894 -> 71;
 //   - the rest: k_gemm_f32.
 int launch_rows_product(mr_ctx *ctx, const float *x, const void *w, int dtype, float *y, int rows, int n, int k) {
     hipStream_t s = ctx->stream;
@@ -1646,21 +1665,16 @@ int launch_rows_product(mr_ctx *ctx, const float *x, const void *w, int dtype, f
     };
     void *ws = nullptr;
     if (terms) {
-        const size_t planes = (dtype == MR_BF16 ? 3 : 2) * (size_t)rows * k * 2;
+        const size_t planes = 3 * (size_t)rows * k * 2;
         const size_t scales = ((size_t)rows * sizeof(float) + 255) / 256 * 256, part = part_bytes(32, 128);
         if (ctx_workspace(ctx, part + planes + scales, &ws) == MR_OK) {
             g.part = part ? (float *)ws : nullptr;
             g.ascale = (float *)((char *)ws + part);
             g.ahl_ws = (_Float16 *)((char *)ws + part + scales);
             g.ahl = g.ahl_ws;
-            if (dtype == MR_BF16) {
-                k_row_split3<<<ceil_div(rows, 4), 256, 0, s>>>(x, k, rows, k, g.ascale, (__bf16 *)g.ahl_ws);
-                launch_hd<GEMM_STORE, kBF16Rows>(s, g);
-            } else {
-                g.wscale = kF16RowsScale;
-                row_split(s, x, k, rows, k, g.ascale, g.ahl_ws);
-                launch_hd<GEMM_STORE, kF16Rows>(s, g);
-            }
+            k_row_split3<<<ceil_div(rows, 4), 256, 0, s>>>(x, k, rows, k, g.ascale, (__bf16 *)g.ahl_ws);
+            if (dtype == MR_BF16) launch_hd<GEMM_STORE, kBF16Rows>(s, g);
+            else launch_hd<GEMM_STORE, kF16Rows>(s, g);
             const hipError_t e = hipGetLastError();
             ctx_release(ctx, ws);   // stream-ordered: later work on this stream reuses it safely
             MR_HIP(e, "linear launch");
@@ -1694,10 +1708,11 @@ int launch_gemm(hipStream_t s, int epilogue, const GemmArgs &g) {
     MR_REQUIRE(((uintptr_t)g.a & 15) == 0 && ((uintptr_t)g.w & 15) == 0 && ((uintptr_t)g.w2 & 15) == 0,
                "gemm: operands must be 16-byte aligned");
     MR_REQUIRE(g.ldc >= g.n, "gemm: output rows too short");
-    MR_REQUIRE(g.wscale <= 0.0f || (g.dtype != MR_F32 && g.ascale && g.ahl_ws && g.wh &&
+    MR_REQUIRE(g.wscale <= 0.0f || (g.dtype == MR_BF16 && g.ascale && g.ahl_ws && g.wh &&
                                      (epilogue != GEMM_SWIGLU || g.wh2) && ((uintptr_t)g.wh & 15) == 0 &&
                                      ((uintptr_t)g.wh2 & 15) == 0),
-               "gemm: FP16 terms need 16-bit weights, their FP16 copies and the row-scale and plane workspaces");
+               "gemm: FP16 terms need BF16 weights, their FP16 copies and the row-scale and plane workspaces");
+    MR_REQUIRE(!g.planes3 || (g.a && g.ascale && g.ahl_ws), "gemm: three planes need their workspaces");
     MR_REQUIRE(ceil_div(g.m, kBM) <= 65535, "gemm: too many rows");
     MR_REQUIRE(!g.c_hl || (epilogue == GEMM_SWIGLU && g.wscale > 0.0f && g.c_scale && ((uintptr_t)g.c_hl & 15) == 0),
                "gemm: an output in FP16 terms needs the FP16-term SwiGLU GEMM and its row scales");

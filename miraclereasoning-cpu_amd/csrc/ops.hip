@@ -600,7 +600,7 @@ int mr_debug_gemm(mr_ctx *ctx, const float *a, const void *w, float *c, float *a
             MR_HIP(ea, "debug gemm workspace");
         }
         g.wh = wh;
-        const int rc = gemm_f16_weight_copy(s, w, MR_BF16, (int64_t)n * k, g.wscale, wh);
+        const int rc = gemm_f16_weight_copy(s, w, (int64_t)n * k, g.wscale, wh);
         if (rc != MR_OK) {
             (void)hipFree(g.ahl_ws);
             (void)hipFree(wh);
@@ -672,7 +672,7 @@ int mr_debug_gemm_grouped(mr_ctx *ctx, const float *a, const void *w, const void
     for (int t = 0; t < mats; ++t)
         for (int z = 0; z < groups; ++z) {
             _Float16 *dst = wh + ((size_t)t * groups + z) * nk;
-            MR_TRY(gemm_f16_weight_copy(s, tab_w[t * groups + z], MR_BF16, nk, scale[t * groups + z], dst));
+            MR_TRY(gemm_f16_weight_copy(s, tab_w[t * groups + z], nk, scale[t * groups + z], dst));
             tab_h[t * groups + z] = dst;
         }
     void **d_w = nullptr, **d_h = nullptr;

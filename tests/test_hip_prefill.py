@@ -64,9 +64,9 @@ def test_batched_workload_geometry_matches_oracle(backend, name, prompt):
 @pytest.mark.parametrize("dtype", ["f16", "f32"])
 @pytest.mark.parametrize("hidden,prompt", [(1024, 5), (1024, 70), (1024, 700), (1000, 70)])
 def test_batched_weight_types_match_token_loop(backend, dtype, hidden, prompt):
-    """F16 weights (FP16 terms over scaled copies) and F32 weights (FP32 products
-    in few tiles, BF16 terms in many), hidden widths in and out of whole
-    k-steps, against the exact token loop."""
+    """F16 weights (BF16 terms, copied into LDS or split in every tile) and F32
+    weights (FP32 products in few tiles, BF16 terms in many), hidden widths in
+    and out of whole k-steps, against the exact token loop."""
     config = {"family": "flashnano-1.5", "vocab_size": 1000, "hidden_size": hidden, "layers": 2, "query_heads": 16,
               "kv_heads": 4, "head_dim": 64, "ffn_dim": 1320, "max_positions": 1024,
               "window": 256, "global_layers": [2], "rope_theta": 1e4, "backend_format": 1}
@@ -81,6 +81,40 @@ def test_batched_weight_types_match_token_loop(backend, dtype, hidden, prompt):
         model = MiracleModel(ModelConfig.from_dict(config), weights, backend=backend, context_length=1024, prefill_mode=mode)
         got[mode] = model.prefill(ids, return_all=True)
         model.close()
+    np.testing.assert_allclose(got["batched"], got["exact"], atol=2e-5, rtol=2e-4)
+
+
+@pytest.mark.parametrize("family,hidden,prompt", [
+    ("flashnano-1.5", 512, 9), ("flashnano-1.5", 512, 70), ("flashnano-1.5", 512, 700), ("flashnano-1.5", 1000, 70),
+    ("flashlighting-2.0", 512, 70)])
+def test_batched_f16_weights_keep_small_activations(backend, family, hidden, prompt):
+    """Two channels of the normalized rows stand 2^26 above the others, where the
+    Q, K, V, gate and up weights are zero: an activation's bits are its own and
+    not its row's largest's, as in the token loop, to the tolerance of the other
+    weight types.  In FP16 terms of the row the others would keep 11 bits."""
+    config = {"family": family, "vocab_size": 300, "hidden_size": hidden, "layers": 2, "query_heads": 8,
+              "kv_heads": 2, "head_dim": 64, "ffn_dim": 1024, "max_positions": 1024, "window": 128,
+              "global_layers": [2], "rope_theta": 1e4, "backend_format": 1}
+    if hidden == 1000:
+        config.update(query_heads=10, head_dim=100)
+    if family == "flashlighting-2.0":
+        from test_hip_model import LIGHT_MID
+        config = dict(LIGHT_MID)
+    weights = synthetic.synthetic_weights(config, 21, "f32")
+    weights = {k: np.array(v, np.float32) for k, v in weights.items()}
+    big = np.array([3, 70])
+    for name, w in weights.items():
+        if name.endswith(("a_norm", "f_norm")):
+            w[big] *= 2.0 ** 26
+        elif name.endswith((".q", ".k", ".v", ".latent", ".gate", ".up")) and w.shape[1] == config["hidden_size"]:
+            w[:, big] = 0
+    weights = {k: v.astype(np.float16) if v.ndim == 2 else v for k, v in weights.items()}
+    ids = synthetic.prompt_ids(config["vocab_size"], prompt, 21)
+    got = {}
+    for mode in ("exact", "batched"):
+        with MiracleModel(ModelConfig.from_dict(config), weights, backend=backend, context_length=1024,
+                          prefill_mode=mode) as model:
+            got[mode] = model.prefill(ids, return_all=True)
     np.testing.assert_allclose(got["batched"], got["exact"], atol=2e-5, rtol=2e-4)
 
 
@@ -280,6 +314,17 @@ def test_batched_heavy_geometry_matches_oracle(backend, parts):
         _heavy_against_oracle(model, cfg, HEAVY_MID, weights, ids, 160, parts)
 
 
+def test_batched_heavy_f16_matches_oracle(backend):
+    """The same with F16 weights (BF16-term products throughout)."""
+    from test_hip_model import HEAVY_MID
+    weights = synthetic.synthetic_weights(HEAVY_MID, 11, "f32")
+    weights = {k: v.astype(np.float16) if v.ndim == 2 else v for k, v in weights.items()}
+    ids = synthetic.prompt_ids(HEAVY_MID["vocab_size"], 100, 11)
+    cfg = ModelConfig.from_dict(HEAVY_MID)
+    with MiracleModel(cfg, weights, backend=backend, context_length=160, prefill_mode="batched") as model:
+        _heavy_against_oracle(model, cfg, HEAVY_MID, weights, ids, 160)
+
+
 def test_batched_heavy_micro_takes_token_loop(backend, golden_dir):
     """The reference's micro heavy model (head dim 4) is outside the batched
     kernels' geometry: under prefill_mode="batched" it takes the token loop and
@@ -316,6 +361,22 @@ def test_batched_lighting_geometry_matches_oracle(backend, slots, parts):
             got = model.prefill(ids, return_all=True)
         np.testing.assert_allclose(got, want, rtol=1e-3, atol=1e-4)
         assert model.generate(list(ids), max_new_tokens=8) == stream
+
+
+@pytest.mark.parametrize("prompt", [5, 90])
+def test_batched_lighting_f16_matches_oracle(backend, prompt):
+    """F16 weights, before and past the first merge, against the oracle."""
+    from oracle.model import OracleModel
+    from test_hip_model import LIGHT_MID
+    config = dict(LIGHT_MID, memory_slots=4)
+    weights = synthetic.synthetic_weights(config, 13, "f32")
+    weights = {k: v.astype(np.float16) if v.ndim == 2 else v for k, v in weights.items()}
+    ids = synthetic.prompt_ids(config["vocab_size"], prompt, 13)
+    ref = OracleModel(config, weights, context_length=128)
+    want = ref.prefill(ids, return_all=True)
+    with MiracleModel(ModelConfig.from_dict(config), weights, backend=backend, context_length=128,
+                      prefill_mode="batched") as model:
+        np.testing.assert_allclose(model.prefill(ids, return_all=True), want, atol=2e-5, rtol=2e-4)
 
 
 def test_batched_lighting_full_prompt_matches_token_loop(backend):

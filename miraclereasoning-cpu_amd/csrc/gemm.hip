@@ -1158,13 +1158,14 @@ void launch_rows_gemv(hipStream_t s, const float *x, const void *w, float *y, in
     else k_rows_gemv<DT, 8><<<grid, 256, 0, s>>>(x, w, y, rows, n, k);
 }
 
-// The K slices k_gemm_f32 gives a product: two workgroups a CU from fewer 64 x
-// 64 tiles than CUs, four k-steps a slice at least.
+// The K slices k_gemm_f32 gives a product that has a workspace for their sums:
+// two workgroups a CU from fewer 64 x 64 tiles than CUs, four k-steps a slice
+// at least.
 int f32_slices(int epi, const GemmArgs &g) {
     const int cols = epi == GEMM_SWIGLU ? 2 * g.n : g.n;
     const int64_t count = (int64_t)ceil_div(cols, 64) * ceil_div(g.m, 64);
     const int nk = ceil_div(g.k, kFK), cus = device_cus();
-    if (!g.part || count > cus) return 1;
+    if (count > cus) return 1;
     const int64_t slices = std::min<int64_t>({(2 * cus + count / 2) / count, std::max(nk / 4, 1),
                                               (int64_t)(kGemmPartFloats / ((size_t)g.m * cols))});
     return ceil_div(nk, ceil_div(nk, (int)std::max<int64_t>(slices, 1)));
@@ -1173,7 +1174,7 @@ int f32_slices(int epi, const GemmArgs &g) {
 template <int DT, int EPI>
 void launch_gemm_f32(hipStream_t s, const GemmArgs &g, int align) {
     const dim3 tiles(ceil_div(EPI == GEMM_SWIGLU ? 2 * g.n : g.n, 64), ceil_div(g.m, 64));
-    const int slices = f32_slices(EPI, g), steps = ceil_div(ceil_div(g.k, kFK), slices);
+    const int slices = g.part ? f32_slices(EPI, g) : 1, steps = ceil_div(ceil_div(g.k, kFK), slices);
     const dim3 grid(tiles.x, tiles.y, slices);
     if (align == 2) k_gemm_f32<DT, 2, EPI><<<grid, 256, 0, s>>>(g, steps);
     else if (align == 1) k_gemm_f32<DT, 1, EPI><<<grid, 256, 0, s>>>(g, steps);
@@ -1404,24 +1405,39 @@ int launch_grouped_dt(hipStream_t s, int epi, const GemmArgs &g, const GemmGroup
 //     for projections whose grid of them still covers every CU, else 128 x 128;
 //     SwiGLU keeps three 128 x 128 workgroups per CU.  A grid of at most one
 //     tile per CU takes two LDS stages, since no other workgroup covers a copy.
+struct HdSlices {
+    int rows = 0;                // of a slice's tiles
+    int slices = 1, steps = 0;   // 1: K whole; k-steps a slice
+};
+
+// The first rule: the slices of a product that has a workspace for their sums.
+HdSlices hd_slices(bool pair, int m, int n, int k) {
+    const int cus = device_cus(), nk = k / kDmaKB, cols = pair ? 2 * n : n;
+    HdSlices r;
+    r.rows = m <= 32 || (m <= 64 && !pair) ? 32 : 64;
+    const int64_t tiles = (int64_t)ceil_div(cols, 128) * ceil_div(m, r.rows);
+    if (tiles > cus) return r;
+    const int64_t room = (int64_t)(kGemmPartFloats / ((size_t)m * cols));
+    const int want = (int)std::min<int64_t>({(cus + cus / 2 + tiles / 2) / tiles, nk / 4, room});
+    if (want >= 2) {
+        r.steps = ceil_div(nk, want);
+        r.slices = ceil_div(nk, r.steps);
+    }
+    return r;
+}
+
 template <int EPI, int SCH = kModelTerms>
 void launch_hd(hipStream_t s, const GemmArgs &h) {
     constexpr bool pair = EPI == GEMM_SWIGLU;
-    const int cus = device_cus(), nk = h.k / kDmaKB, cols = pair ? 2 * h.n : h.n;
+    const int cus = device_cus(), cols = pair ? 2 * h.n : h.n;
     const int gx = ceil_div(cols, 128);
-    const bool low = h.m <= 32 || (h.m <= 64 && !pair);
-    const int64_t tiles = (int64_t)gx * ceil_div(h.m, low ? 32 : 64);
-    if (h.part && tiles <= cus) {
-        const int64_t room = (int64_t)(kGemmPartFloats / ((size_t)h.m * cols));
-        const int want = (int)std::min<int64_t>({(cus + cus / 2 + tiles / 2) / tiles, nk / 4, room});
-        if (want >= 2) {
-            const int steps = ceil_div(nk, want), slices = ceil_div(nk, steps);
-            const dim3 grid(gx, ceil_div(h.m, low ? 32 : 64), slices);
-            if (low) k_gemm_hd_split<EPI, 4, kDmaKB, 2, 2, 1, SCH><<<grid, 256, 0, s>>>(h, steps);
-            else k_gemm_hd_split<EPI, 4, kDmaKB, 2, 2, 2, SCH><<<grid, 256, 0, s>>>(h, steps);
-            finish_slices<EPI, SCH>(s, h, slices);
-            return;
-        }
+    const HdSlices cut = hd_slices(pair, h.m, h.n, h.k);
+    if (h.part && cut.slices > 1) {
+        const dim3 grid(gx, ceil_div(h.m, cut.rows), cut.slices);
+        if (cut.rows == 32) k_gemm_hd_split<EPI, 4, kDmaKB, 2, 2, 1, SCH><<<grid, 256, 0, s>>>(h, cut.steps);
+        else k_gemm_hd_split<EPI, 4, kDmaKB, 2, 2, 2, SCH><<<grid, 256, 0, s>>>(h, cut.steps);
+        finish_slices<EPI, SCH>(s, h, cut.slices);
+        return;
     }
     const dim3 grid64(gx, ceil_div(h.m, 64));
     const int64_t tiles64 = (int64_t)grid64.x * grid64.y;
@@ -1503,7 +1519,7 @@ int launch_dt(hipStream_t s, int epi, const GemmArgs &g) {
     // (176 tiles) 175 -> 64.7.  With K whole the term products
     // stay: their error against FP64 is the smaller one (1024 x 2816, rms:
     // terms 8.2e-7, here whole 9.5e-7, in two slices 5.5e-7, in ten 3.9e-7).
-    if (DT == MR_F32 && f32_slices(epi, g) > 1) {
+    if (DT == MR_F32 && g.part && f32_slices(epi, g) > 1) {
         switch (epi) {
             case GEMM_STORE: launch_gemm_f32<DT, GEMM_STORE>(s, g, 2); break;
             case GEMM_RESIDUAL: launch_gemm_f32<DT, GEMM_RESIDUAL>(s, g, 2); break;
@@ -1659,14 +1675,13 @@ int launch_rows_product(mr_ctx *ctx, const float *x, const void *w, int dtype, f
         MR_LAUNCHED("linear launch");
         return MR_OK;
     }
-    const auto part_bytes = [&](int tile_rows, int tile_cols) {   // a split product's sums
-        const int64_t tiles = (int64_t)ceil_div(n, tile_cols) * ceil_div(rows, tile_rows);
-        return tiles <= device_cus() ? kGemmPartFloats * sizeof(float) : (size_t)0;
+    const auto part_bytes = [&](int slices) {   // the sums of a product cut into slices
+        return slices > 1 ? ((size_t)slices * rows * n * sizeof(float) + 255) / 256 * 256 : (size_t)0;
     };
     void *ws = nullptr;
     if (terms) {
         const size_t planes = 3 * (size_t)rows * k * 2;
-        const size_t scales = ((size_t)rows * sizeof(float) + 255) / 256 * 256, part = part_bytes(32, 128);
+        const size_t scales = ((size_t)rows * sizeof(float) + 255) / 256 * 256, part = part_bytes(hd_slices(false, rows, n, k).slices);
         if (ctx_workspace(ctx, part + planes + scales, &ws) == MR_OK) {
             g.part = part ? (float *)ws : nullptr;
             g.ascale = (float *)((char *)ws + part);
@@ -1683,7 +1698,7 @@ int launch_rows_product(mr_ctx *ctx, const float *x, const void *w, int dtype, f
     }
     // no room for the terms, or a product they do not take (K then stays
     // whole where there is no room for its slices' sums either)
-    const size_t part = part_bytes(64, 64);
+    const size_t part = part_bytes(f32_slices(GEMM_STORE, g));
     if (part && ctx_workspace(ctx, part, &ws) == MR_OK) g.part = (float *)ws;
     const int align = !x16 || k % 4 || (dtype == MR_F32 ? !w16 : ((uintptr_t)w & 7) != 0) ? 0
                       : dtype == MR_F32 || (k % 8 == 0 && w16)                          ? 2

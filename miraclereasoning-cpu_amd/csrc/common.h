@@ -49,6 +49,10 @@ struct mr_ctx {
     // size -> free device blocks (all blocks of one size class)
     std::unordered_map<size_t, std::vector<void *>> free_blocks;
     std::unordered_map<void *, size_t> live;   // block -> size class
+    // the block of ctx_workspace, as large as the largest call needed
+    void *work = nullptr;
+    size_t work_bytes = 0;
+    bool work_taken = false;
     // The caller's reference plus one per live model; the stream and the
     // blocks are released when the last one goes (mr_ctx_destroy and
     // mr_model_destroy may then come in either order).
@@ -60,9 +64,12 @@ namespace mr {
 
 int ctx_alloc(mr_ctx *ctx, size_t bytes, void **ptr);
 void ctx_release(mr_ctx *ctx, void *ptr);
-// A block for one call's intermediate values (release it after the launches):
-// a power of two of bytes, so that calls of many sizes share few blocks.
+// A block for one call's intermediate values (give it back with ctx_release
+// after the launches).  The context holds one for all calls, which grows by
+// eighths of a power of two: a block a size would add up over a program's sizes.
 int ctx_workspace(mr_ctx *ctx, size_t bytes, void **ptr);
+// Returns every block that no call and no tensor holds to the device.
+void ctx_trim(mr_ctx *ctx);
 void ctx_retain(mr_ctx *ctx);
 void ctx_unref(mr_ctx *ctx);
 

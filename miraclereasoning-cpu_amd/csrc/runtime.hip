@@ -37,12 +37,7 @@ int ctx_alloc(mr_ctx *ctx, size_t bytes, void **ptr) {
     void *p = nullptr;
     hipError_t e = hipMalloc(&p, cls);
     if (e != hipSuccess) {
-        // Give cached blocks back and try once more.
-        hipStreamSynchronize(ctx->stream);
-        for (auto &kv : ctx->free_blocks)
-            for (void *q : kv.second) hipFree(q);
-        ctx->free_blocks.clear();
-        (void)hipGetLastError();
+        ctx_trim(ctx);
         e = hipMalloc(&p, cls);
         if (e != hipSuccess) {
             (void)hipGetLastError();   // not the next launch's error
@@ -55,13 +50,42 @@ int ctx_alloc(mr_ctx *ctx, size_t bytes, void **ptr) {
     return MR_OK;
 }
 
+void ctx_trim(mr_ctx *ctx) {
+    hipStreamSynchronize(ctx->stream);
+    for (auto &kv : ctx->free_blocks)
+        for (void *q : kv.second) hipFree(q);
+    ctx->free_blocks.clear();
+    if (ctx->work && !ctx->work_taken) {
+        hipFree(ctx->work);
+        ctx->work = nullptr;
+        ctx->work_bytes = 0;
+    }
+    (void)hipGetLastError();
+}
+
 int ctx_workspace(mr_ctx *ctx, size_t bytes, void **ptr) {
-    size_t c = (size_t)64 << 10;
-    while (c < bytes) c *= 2;
-    return ctx_alloc(ctx, c, ptr);
+    if (ctx->work_taken) return ctx_alloc(ctx, bytes, ptr);
+    if (bytes > ctx->work_bytes) {
+        size_t step = (size_t)8 << 10;
+        while (8 * step < bytes) step *= 2;
+        const size_t want = (bytes + step - 1) / step * step;
+        if (ctx->work) hipFree(ctx->work);   // waits for the calls that use it
+        ctx->work = nullptr;
+        ctx->work_bytes = 0;
+        MR_TRY(ctx_alloc(ctx, want, &ctx->work));
+        ctx->live.erase(ctx->work);
+        ctx->work_bytes = want;
+    }
+    ctx->work_taken = true;
+    *ptr = ctx->work;
+    return MR_OK;
 }
 
 void ctx_release(mr_ctx *ctx, void *ptr) {
+    if (ptr && ptr == ctx->work) {
+        ctx->work_taken = false;
+        return;
+    }
     auto it = ctx->live.find(ptr);
     if (it == ctx->live.end()) return;
     ctx->free_blocks[it->second].push_back(ptr);
@@ -77,6 +101,7 @@ void ctx_unref(mr_ctx *ctx) {
     for (auto &kv : ctx->free_blocks)
         for (void *p : kv.second) hipFree(p);
     for (auto &kv : ctx->live) hipFree(kv.first);
+    if (ctx->work) hipFree(ctx->work);
     hipStreamDestroy(ctx->stream);
     delete ctx;
 }

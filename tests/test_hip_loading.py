@@ -189,3 +189,26 @@ def test_freed_buffers_are_recycled_within_bounds():
     del other
     b.close()
     assert b._pooled == 0
+
+
+def _free_bytes(b):
+    import ctypes as C
+    free, total = C.c_size_t(), C.c_size_t()
+    assert b.lib.hipMemGetInfo(C.byref(free), C.byref(total)) == 0   # of the runtime the library is linked to
+    return free.value
+
+
+def test_workspace_is_one_block_as_large_as_needed():
+    """Linears of growing and shrinking sizes leave one workspace, of the
+    largest call's size, not one a size."""
+    from miracle_hip import HIPBackend
+    b = HIPBackend()
+    w = b.upload_weight(np.ones((256, 2048), np.float16))
+    xs = [b.upload(np.ones((rows, 2048), np.float32)) for rows in (8192, 700, 1400, 2600, 5100, 8192)]
+    b.read(b.linear(xs[0], w))
+    free = _free_bytes(b)
+    for x in xs:
+        np.testing.assert_array_equal(b.read(b.linear(x, w)), np.full((x.shape[0], 256), 2048, np.float32))
+    # the outputs' own blocks: 1 MiB a thousand rows
+    assert _free_bytes(b) > free - (32 << 20)
+    b.close()

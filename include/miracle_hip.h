@@ -279,6 +279,11 @@ MR_API int mr_model_time_kernel(mr_model *model, int which, int reps, float *avg
  * model.py:298-311).  Not a counterpart of any reference function. */
 MR_API int mr_debug_fail_next(mr_ctx *ctx);
 
+/* Test hook: the next device allocation of a model of this context finds no
+ * memory at first (the library then returns the context's cached blocks to the
+ * device and asks again).  Not a counterpart of any reference function. */
+MR_API int mr_debug_fail_alloc(mr_ctx *ctx);
+
 /* Test hook: the status check after the model's next persistent step reports
  * MR_ERR_TIMEOUT as if a wait had given up (the host-side half of the
  * timeout path: the error, the poisoned model, the switch to MR_STEP_GRAPH at

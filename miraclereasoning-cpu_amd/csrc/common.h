@@ -49,6 +49,7 @@ struct mr_ctx {
     // size -> free device blocks (all blocks of one size class)
     std::unordered_map<size_t, std::vector<void *>> free_blocks;
     std::unordered_map<void *, size_t> live;   // block -> size class
+    bool fail_alloc = false;                   // test hook: the next model allocation finds no memory
     // the block of ctx_workspace, as large as the largest call needed
     void *work = nullptr;
     size_t work_bytes = 0;

@@ -350,8 +350,14 @@ __global__ void __launch_bounds__(256) k_rows_rms(const void *x, int dt, float *
 
 // ------------------------------------------------------------------ host helpers
 int device_alloc(mr_model *m, size_t bytes, void **p) {
-    MR_HIP(hipMalloc(p, bytes ? bytes : 16), "allocate model buffer");
-    (void)m;
+    hipError_t e = m->ctx->fail_alloc ? hipErrorOutOfMemory : hipMalloc(p, bytes ? bytes : 16);
+    m->ctx->fail_alloc = false;
+    if (e != hipSuccess) {   // what the context only keeps for later calls goes first
+        ctx_trim(m->ctx);
+        e = hipMalloc(p, bytes ? bytes : 16);
+        if (e != hipSuccess) (void)hipGetLastError();   // not the next launch's error
+    }
+    MR_HIP(e, "allocate model buffer");
     return MR_OK;
 }
 

@@ -230,4 +230,10 @@ int mr_debug_fail_next(mr_ctx *ctx) {
     return MR_OK;
 }
 
+int mr_debug_fail_alloc(mr_ctx *ctx) {
+    MR_REQUIRE(ctx, "mr_debug_fail_alloc: null context");
+    ctx->fail_alloc = true;
+    return MR_OK;
+}
+
 }  // extern "C"

@@ -100,6 +100,7 @@ _SIGNATURES = {
     "mr_model_choices": [_P, _P, C.c_int64, C.POINTER(_i)],
     "mr_model_time_kernel": [_P, _i, _i, C.POINTER(C.c_float)],
     "mr_debug_fail_next": [_P],
+    "mr_debug_fail_alloc": [_P],
     "mr_debug_step_timeout": [_P],
     "mr_debug_gemm": [_P, _P, _P, _P, _P, _i, _i, _i, _i],
     "mr_debug_gemm_grouped": [_P, _P, _P, _P, _P, C.POINTER(C.c_int), _i, _i, _i, _i, _i],

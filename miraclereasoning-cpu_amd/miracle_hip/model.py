@@ -101,6 +101,7 @@ class Engine:
         self.backend, self.lib, self.config = backend, backend.lib, config
         if backend.ctx is None:
             raise HIPError("create model failed: the backend is closed")
+        backend._empty_pool()   # into the library's blocks, which a model's buffers may claim
         handle = C.c_void_p()
         desc = model_desc(config, context_length)
         _check(self.lib.mr_model_create(backend.ctx, C.byref(desc), C.byref(handle)), "create model")

@@ -198,6 +198,29 @@ def _free_bytes(b):
     return free.value
 
 
+def test_model_buffers_claim_cached_blocks():
+    """A model's allocation that finds no memory takes back what the context
+    only keeps: freed tensors of both pools and the operations' workspace."""
+    from miracle_hip import HIPBackend
+    bundle = presets.micro("flashnano-1.7")
+    b = HIPBackend()
+    x, w = b.upload(np.ones((4096, 2048), np.float32)), b.upload_weight(np.ones((2048, 2048), np.float16))
+    b.read(b.linear(x, w))                    # its workspace: three planes of x, 48 MiB
+    tensor = b.empty((1 << 28,))              # 1 GiB, past the pool: the library's free blocks
+    del x, w, tensor
+    free = _free_bytes(b)
+    assert b.lib.mr_debug_fail_alloc(b.ctx) == 0
+    with MiracleModel(ModelConfig.from_dict(bundle), synthetic.micro_weights(bundle), backend=b,
+                      context_length=32) as model:
+        assert not b._pool
+        model.prefill([1, 2, 3])
+        # a gibibyte of blocks and the workspace came back, less the model's own few buffers
+        assert _free_bytes(b) > free + (1 << 30) + (16 << 20)
+    y = b.read(b.linear(b.upload(np.ones((40, 128), np.float32)), b.upload_weight(np.ones((8, 128), np.float16))))
+    np.testing.assert_array_equal(y, np.full((40, 8), 128, np.float32))
+    b.close()
+
+
 def test_workspace_is_one_block_as_large_as_needed():
     """Linears of growing and shrinking sizes leave one workspace, of the
     largest call's size, not one a size."""

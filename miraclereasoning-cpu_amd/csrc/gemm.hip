@@ -148,16 +148,6 @@ __device__ __forceinline__ void split2h(float x, _Float16 &hi, _Float16 &lo) {
     lo = (_Float16)(x - (float)hi);
 }
 
-// Eight halves as two BF16 terms each (exact: 11 bits fit in 8 + 8).
-__device__ __forceinline__ void split_f16(const f16x8 &f, bf16x8 &hi, bf16x8 &lo) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const float x = (float)f[e];
-        hi[e] = (__bf16)x;
-        lo[e] = (__bf16)(x - (float)hi[e]);
-    }
-}
-
 template <int DT>
 __device__ __forceinline__ void store_w(__bf16 (*bs)[kBN][kPitch], const WRegs<DT> &r) {
     const int tid = threadIdx.x;
@@ -171,8 +161,14 @@ __device__ __forceinline__ void store_w(__bf16 (*bs)[kBN][kPitch], const WRegs<D
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int idx = tid + kThreads * i;
+            const f16x8 f = __builtin_bit_cast(f16x8, r.v[i]);
             bf16x8 h, l;
-            split_f16(__builtin_bit_cast(f16x8, r.v[i]), h, l);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float x = (float)f[e];
+                h[e] = (__bf16)x;
+                l[e] = (__bf16)(x - (float)h[e]);
+            }
             *(bf16x8 *)&bs[0][idx >> 2][(idx & 3) * 8] = h;
             *(bf16x8 *)&bs[1][idx >> 2][(idx & 3) * 8] = l;
         }
@@ -213,7 +209,7 @@ __device__ __forceinline__ f32x4 mfma(const f16x8 &a, const f16x8 &b, const f32x
 // keep them relative to the row's largest only); a BF16 weight is one term, an
 // F16 weight two BF16 terms split in registers (exact, subnormals too, which
 // the FP16 matrix cores would multiply at fewer bits).  4096 rows of 5632 x
-// 2048 take 283 us by BF16 weights (three products a weight) and 437 by F16
+// 2048 take 277 us by BF16 weights (three products a weight) and 423 by F16
 // weights (five); in two FP16 planes 213.
 // Splitting a value into terms turns an infinity into inf - inf, and a scaled
 // row can overflow where its FP32 products would not, so STORE products of
@@ -233,6 +229,24 @@ struct Terms<kModelTerms> {
     static constexpr int kPlanes = 2, kWeightTerms = 1;
     static constexpr bool kRecompute = false;
 };
+
+// Eight halves as two BF16 terms each, exact (11 bits fit in 8 + 3): the upper
+// halves of the FP32 value and of what they leave, by moves of whole 16-bit
+// words (by conversions to BF16: 333 rows of 5632 x 2048 82.5 us against 79.1,
+// 4096 rows 450 against 423).
+__device__ __forceinline__ void split_f16(const f16x8 &f, bf16x8 &hi, bf16x8 &lo) {
+    u32x4 h, l;
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+        const float x0 = (float)f[e], x1 = (float)f[e + 1];
+        const unsigned u0 = __float_as_uint(x0), u1 = __float_as_uint(x1);
+        const float r0 = x0 - __uint_as_float(u0 & 0xffff0000u), r1 = x1 - __uint_as_float(u1 & 0xffff0000u);
+        h[e / 2] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
+        l[e / 2] = __builtin_amdgcn_perm(__float_as_uint(r1), __float_as_uint(r0), 0x07060302u);
+    }
+    hi = __builtin_bit_cast(bf16x8, h);
+    lo = __builtin_bit_cast(bf16x8, l);
+}
 
 // Output (row, col) of g from its FP32 rows and stored weights, k in order.
 template <int SCH>
@@ -656,11 +670,17 @@ __device__ __forceinline__ void gemm_tile_hd(const GemmArgs &g, int m0, int n0, 
         }
     };
 
-    f32x4 acc[MI][NI];
+    // With two weight terms the four smaller term pairs have sums of their own,
+    // so a k-step rounds the large sum once, not five times (the MLP of 50 rows of
+    // 1024 x 2816: 9.9e-8 off float64 in one sum, 6.0e-8 in two).
+    constexpr int U = T > 1 ? 2 : 1;
+    f32x4 acc[U][MI][NI];
 #pragma unroll
-    for (int mi = 0; mi < MI; ++mi)
+    for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni) acc[u][mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
     static_assert(S == 1 || S == 2, "stages");
     issue(kt0, 0);
     int stage = 0;
@@ -694,7 +714,7 @@ __device__ __forceinline__ void gemm_tile_hd(const GemmArgs &g, int m0, int n0, 
                         if (o - q >= 0 && o - q < P)
 #pragma unroll
                             for (int ni = 0; ni < NI; ++ni)
-                                acc[mi][ni] = mfma(term[o - q], bf[q][ni], acc[mi][ni]);
+                                acc[o ? U - 1 : 0][mi][ni] = mfma(term[o - q], bf[q][ni], acc[o ? U - 1 : 0][mi][ni]);
             }
         }
         if (S == 1 && kt + 1 < kt1) {
@@ -703,8 +723,13 @@ __device__ __forceinline__ void gemm_tile_hd(const GemmArgs &g, int m0, int n0, 
         }
         stage ^= S - 1;
     }
+    if constexpr (U == 2)
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni) acc[0][mi][ni] += acc[1][mi][ni];
     const float inv_w = 1.0f / g.wscale;
-    gemm_store<EPI, NI, WN, MI, SCH>(g, m0, n0, acc, [&](int row) { return (1.0f / g.ascale[row]) * inv_w; }, part);
+    gemm_store<EPI, NI, WN, MI, SCH>(g, m0, n0, acc[0], [&](int row) { return (1.0f / g.ascale[row]) * inv_w; }, part);
 }
 
 constexpr int kDmaKB = 64, kDmaBlocksPerCU = 3;
@@ -1496,7 +1521,7 @@ int launch_dt(hipStream_t s, int epi, const GemmArgs &g) {
     // F16 weights as stored by three BF16 planes of the rows: the products of
     // k_gemm<MR_F16> in its order, with K in slices and operands copied into LDS
     // (prefill of four layers of flashnano-1.7, us by k_gemm -> here: 45 tokens
-    // 2582 -> 667, 217 2641 -> 1102, 1000 3164 -> 2429, 4096 7368 -> 6997).
+    // 2582 -> 678, 217 2641 -> 1067, 1000 3164 -> 2374, 1900 4257 -> 3802).
     if constexpr (DT == MR_F16) {
         if (g.planes3 && !g.ldw && dma_tile_fits(g)) {
             GemmArgs h = g;
@@ -1655,7 +1680,7 @@ int gemm_f16_weight_copy(hipStream_t s, const void *w, int64_t count, float scal
 //   - 16-bit weights, K a multiple of 64, 16-byte aligned: x in three BF16
 //     terms once (k_row_split3), then the LDS-copy tiles over the weights as
 //     stored.  Against 64 x 64 FP32 tiles: 333 rows of 5632 x 2048 BF16 346 ->
-//     46 us, of 2048 x 5632 894 -> 47; F16 348 -> 85 and 894 -> 71;
+//     46 us, of 2048 x 5632 894 -> 47; F16 348 -> 79 and 894 -> 66;
 //   - the rest: k_gemm_f32.
 int launch_rows_product(mr_ctx *ctx, const float *x, const void *w, int dtype, float *y, int rows, int n, int k) {
     hipStream_t s = ctx->stream;

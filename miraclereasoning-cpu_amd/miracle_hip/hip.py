@@ -222,7 +222,9 @@ class Tensor:
 
 # Bytes of freed buffers a backend keeps by size for its next tensors, on top of
 # the library's own recycling: the calls into it for a buffer and back cost
-# about a fifth of enqueueing an operation.
+# about a fifth of enqueueing an operation.  Past them the sizes pooled first
+# go back (one that is still in use returns with its next release), so sizes
+# that a program no longer uses do not fill it for good.
 _POOL_BYTES = 64 << 20
 
 
@@ -304,6 +306,18 @@ class HIPBackend:
         if self._pooled + nbytes <= _POOL_BYTES:
             self._pooled += nbytes
             self._pool.setdefault(nbytes, []).append(handle)
+            return
+        if nbytes <= _POOL_BYTES:   # the oldest sizes make room
+            self._pool.setdefault(nbytes, []).append(handle)
+            self._pooled += nbytes
+            while self._pooled > _POOL_BYTES:
+                oldest, kept = next(iter(self._pool.items()))
+                if kept:
+                    self._pooled -= oldest
+                    handle = kept.pop()
+                    self.lib.mr_free(self.ctx, handle)
+                else:
+                    del self._pool[oldest]
         else:
             self.lib.mr_free(self.ctx, handle)
 

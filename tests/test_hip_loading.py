@@ -191,6 +191,31 @@ def test_freed_buffers_are_recycled_within_bounds():
     assert b._pooled == 0
 
 
+def test_full_pool_gives_up_its_oldest_sizes():
+    """Sizes that do not come back fill the pool once; after that a new size is
+    recycled all the same, the stale ones go first and the bound holds."""
+    from miracle_hip import HIPBackend
+    from miracle_hip import hip as module
+    b = HIPBackend()
+    for i in range(20):                       # 20 x 4 MiB and some: more than the pool
+        del_me = b.empty(((1 << 20) + 64 * i,))
+        del del_me
+    assert module._POOL_BYTES - (5 << 20) < b._pooled <= module._POOL_BYTES
+    first, last = 4 * (1 << 20), 4 * ((1 << 20) + 64 * 19)
+    assert not b._pool.get(first) and len(b._pool[last]) == 1
+    handle = b.empty((1000,)).handle
+    assert b._pool[4000] == [handle]
+    more = [b.empty((2 << 20,)) for _ in range(6)]
+    del more
+    assert b._pool[4000] == [handle] and len(b._pool[8 << 20]) == 6 and b._pooled <= module._POOL_BYTES
+    assert b._pooled == sum(size * len(kept) for size, kept in b._pool.items())
+    huge = b.empty((17 << 20,))               # past the pool's bytes: it displaces nothing
+    pooled = b._pooled
+    del huge
+    assert b._pooled == pooled and b._pool[4000] == [handle]
+    b.close()
+
+
 def _free_bytes(b):
     import ctypes as C
     free, total = C.c_size_t(), C.c_size_t()

@@ -4,6 +4,7 @@ covers them; the backend refuses to run without a gfx950 GPU (no fallback);
 weights are validated before any device work."""
 import ctypes
 import re
+import subprocess
 from pathlib import Path
 
 import numpy as np
@@ -12,7 +13,9 @@ import pytest
 from miracle_hip import HIPBackend, HIPError, MiracleModel, ModelConfig, presets, synthetic
 from miracle_hip import hip
 
-HEADER = Path(__file__).resolve().parents[1] / "include" / "miracle_hip.h"
+ROOT = Path(__file__).resolve().parents[1]
+HEADER = ROOT / "include" / "miracle_hip.h"
+CSRC = ROOT / "miraclereasoning-cpu_amd" / "csrc"
 
 
 def declared():
@@ -34,6 +37,13 @@ def test_library_exports_every_declared_symbol():
 def test_binding_covers_every_declared_symbol():
     covered = set(hip._SIGNATURES) | {"mr_last_error"}
     assert set(declared()) <= covered, set(declared()) - covered
+
+
+@pytest.mark.parametrize("header", sorted(p.name for p in CSRC.glob("*.h")) + ["../../include/miracle_hip.h"])
+def test_build_follows_every_header(header):
+    """A changed header makes the library out of date (make -q: 1)."""
+    run = subprocess.run(["make", "-q", "-W", header, "-C", str(CSRC)], capture_output=True, text=True)
+    assert run.returncode == 1, (run.returncode, run.stderr)
 
 
 def test_descriptor_layout_matches_header():

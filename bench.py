@@ -14,8 +14,8 @@ Prints one JSON line.  `value` is decode tokens/s with weights and KV cache
 resident in HBM.  `roofline` is for the decode step, timed live with HIP
 events (algorithmic bytes B(P) averaged over the decode positions): the captured
 graph of a token (the default at this size) or the persistent step kernel (one
-launch = one token); in the eager mode for the fused RMSNorm + gate/up GEMV +
-SwiGLU (46.2 MB per launch).
+launch = one token); in the eager mode of the GQA families for the fused RMSNorm +
+gate/up GEMV + SwiGLU (46.2 MB per launch).
 `cpu_baseline` times the oracle (a C restatement of the
 reference's OpenCL kernels, FP32 weights resident, the reference's token loop)
 on this host's cores for a bounded sample of steps at the GPU's decode positions
@@ -427,10 +427,11 @@ def main():
                 "achieved": round(avg_bytes / (step_ms * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(avg_bytes / (step_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4), "traffic": traffic,
                 "traffic_measured": measured, "algorithmic_bytes": int(avg_bytes), "avg_ms": round(step_ms, 5)}
-    elif step_mode == "graph":
-        # the graph-captured step (many small kernels) as one unit
+    elif step_mode == "graph" or not gqa:
+        # the step of many small kernels as one unit
         step_ms = device_ms / args.steps
-        roof = {"kernel": f"graph-captured decode step ({cfg.layers} layers + LM head + greedy choice)",
+        how = "graph-captured" if step_mode == "graph" else "eager"
+        roof = {"kernel": f"{how} decode step ({cfg.layers} layers + LM head + greedy choice)",
                 "bound": "hbm", "achieved": round(avg_bytes / (step_ms * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": round(avg_bytes / (step_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4), "traffic": None,
                 "algorithmic_bytes": int(avg_bytes), "avg_ms": round(step_ms, 5)}

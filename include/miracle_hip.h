@@ -219,9 +219,9 @@ MR_API int mr_model_forward(mr_model *model, const int32_t *ids, int n, int flag
 MR_API int mr_model_generate_greedy(mr_model *model, int max_new, int eos, int32_t *tokens, int *produced);
 
 /* How a token step runs.  A model starts in MR_STEP_PERSISTENT where it streams
- * at most 64 MiB of weights a step, else in MR_STEP_GRAPH, which is faster
- * there.  MR_STEP_PERSISTENT: one kernel launch per
- * step walks the whole layer stack, one workgroup per CU (used when every
+ * at most 64 MiB of weights a step, which needs no capture on the first tokens,
+ * else in MR_STEP_GRAPH, the faster of the two over a longer sequence of any
+ * model measured.  MR_STEP_PERSISTENT: one kernel launch per step walks the whole layer stack, one workgroup per CU (used when every
  * phase fits it; otherwise the model runs MR_STEP_GRAPH).  Its workgroups wait
  * on each other's results, so they must all be resident at once: a plain
  * launch whose grid equals the CU count and whose registers fill a CU places

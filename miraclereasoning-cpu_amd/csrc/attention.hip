@@ -203,16 +203,15 @@ bool tiled_dim(int d) { return d == 32 || d == 64 || d == 128; }
 
 bool tiled(const AttnStepArgs &a) { return tiled_dim(a.dim) && a.heads / a.kv_heads <= kMaxG; }
 
-// The tiled calls are bounded by the LDS of a unit and of one workgroup merging
-// every query head of a KV head.
+// The tiled calls that are accepted: those whose unit, and whose splits merged
+// for every query head of a KV head by one workgroup, fit 64 KiB of LDS (15
+// query heads a KV head with up to 33 splits, fewer heads with more).  The
+// kernels need less, a merge workgroup taking one query head, but what is
+// refused here has always been.
 size_t lds_tiled(int G, int d, int splits) {
-    int main = 0, comb = 0;
-    switch (d) {
-        case 32: main = unit_lds_floats<32>(G); comb = combine_lds_floats<32>(G, splits); break;
-        case 64: main = unit_lds_floats<64>(G); comb = combine_lds_floats<64>(G, splits); break;
-        default: main = unit_lds_floats<128>(G); comb = combine_lds_floats<128>(G, splits); break;
-    }
-    return (size_t)std::max(main, comb) * sizeof(float);
+    const int unit = d == 32 ? unit_lds_floats<32>(G) : d == 64 ? unit_lds_floats<64>(G) : unit_lds_floats<128>(G);
+    const int merge = 2 * splits * G + G + 4 * kThreads * G;
+    return (size_t)std::max(unit, merge) * sizeof(float);
 }
 
 size_t lds_generic(int G, int d, int split_len) { return (size_t)(G * d + 2 * d + G * split_len + 4) * sizeof(float); }

@@ -395,11 +395,6 @@ __device__ __forceinline__ void merge_weights(float *w, const float *lv, float *
     __syncthreads();
 }
 
-template <int D, int NT = kThreads>
-__host__ __device__ constexpr int combine_lds_floats(int G, int splits) {
-    return 2 * splits * G + G + (NT / (D / 4)) * G * D;
-}
-
 // The persistent kernel's merge: the partials of the `active` splits of unit
 // group v (AttnStepArgs::head_groups) are cells of epoch io.ep_out.  Thread
 // (gh, j4, sg) sums float4

@@ -972,12 +972,13 @@ int setup_persistent(mr_model *m) {
            "upload step program");
     m->persistent_ok = true;
     // Which step a model starts with, unless the caller has chosen.  The
-    // per-layer kernels' graph is the faster step (a greedy token of the 24
-    // layers of 2048 at position 300: 871 us against 1169; four layers of 1024:
-    // 125 against 178), so models that stream more than kPersistentBytes of
-    // weights a step run it.  Below, both are bound by latency (four layers of
-    // 256: 105 against 149), and the one-launch step, which needs no capture on
-    // its first tokens (250 us), stays the default.
+    // per-layer kernels' graph was the faster step of every model measured (a
+    // greedy token of the 24 layers of 2048 at position 300: 871 us against 1169;
+    // four layers of 1024: 125 against 178; four of 256: 105 against 149), and
+    // models that stream more than kPersistentBytes of weights a step start with
+    // it.  Smaller ones start with the one-launch step, which needs no capture
+    // (250 us, once a model): a choice for the first half dozen tokens that no
+    // measured crossing backs past them; mr_model_set_step_mode has the other.
     constexpr int64_t kPersistentBytes = (int64_t)64 << 20;
     const auto bytes = [](const Weight &w) { return w.rows * w.cols * dtype_bytes(w.dtype); };
     int64_t streamed = bytes(d.tie_embeddings ? m->embed : m->output);

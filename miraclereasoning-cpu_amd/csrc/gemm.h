@@ -49,9 +49,10 @@ struct GemmArgs {
     // into planes [hi: m x n | lo: m x n] of c_hl.
     _Float16 *c_hl = nullptr;
     const float *c_scale = nullptr;
-    // Optional workspace of kGemmPartFloats floats: FP16-term and FP32 products
-    // with too few output tiles for the device may then cut K into slices, each its
-    // own workgroups, and sum them in order.
+    // Optional workspace of kGemmPartFloats floats (the most that the slices'
+    // sums take): term products by copied tiles and FP32 products, with too few
+    // output tiles for the device, may then cut K into slices, each its own
+    // workgroups, and sum them in order.
     float *part = nullptr;
     // Host only, optional: a product cut into slices then leaves its slices'
     // sums in `part` (slice z's row r at (z m + r) n floats) and their count

@@ -311,11 +311,10 @@ class HIPBackend:
             self._pool.setdefault(nbytes, []).append(handle)
             self._pooled += nbytes
             while self._pooled > _POOL_BYTES:
-                oldest, kept = next(iter(self._pool.items()))
-                if kept:
+                oldest = next(iter(self._pool))   # a key: no container is made that could start a collection
+                if self._pool[oldest]:
                     self._pooled -= oldest
-                    handle = kept.pop()
-                    self.lib.mr_free(self.ctx, handle)
+                    self.lib.mr_free(self.ctx, self._pool[oldest].pop())
                 else:
                     del self._pool[oldest]
         else:
